@@ -1,7 +1,8 @@
 """The FFT building blocks of the PME transforms (fft_core.hpp: radix 2, 3, 4,
 5, 8 butterflies and Stockham stages, run here through their host path with
-the device kernels' compile-time plans) against a naive DFT, for every grid
-length with a specialized kernel and both directions.  CPU only; needs hipcc."""
+the device kernels' compile-time plans) and the two-factor transforms
+(fft_reg.hpp) against a naive DFT, in FP32 also whether their error scales the
+result.  CPU only; needs hipcc."""
 import os
 import shutil
 import subprocess

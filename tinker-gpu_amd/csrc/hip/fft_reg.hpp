@@ -10,6 +10,17 @@
 // with one exchange of A between them.  Products are rounded once into fused
 // multiply-adds written out by hand and contraction is off, so a transform
 // gives the same bits in every kernel that uses it.
+//
+// The constants of the R-point DFTs are hi + lo pairs in FP32.  Each is used for
+// whole frequencies, so its rounding scales them and does not average out over
+// the grid: with constants of 24 bits a 3D transform came out between 9e-8 too
+// small (lengths 96, 144) and 9e-8 too large (100), and the reciprocal energy,
+// which goes through it twice, with it.  Now -3e-8 (64) to 1e-8, from the
+// twiddles, which stay at 24 bits (they are many and mostly average; with low
+// parts 2e-9, but a step of 12,288 atoms 2 % longer), at the same speed (120^3
+// 42.9 -> 43.6 us, dynamics within 0.4 %).  A product with a low part is added
+// to a product with a high part and not to a value of 24 bits, which would
+// swallow it.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -64,6 +75,33 @@ __host__ __device__ __forceinline__ Cplx<real> cmul_fma(Cplx<real> a, Cplx<real>
   return {t9_fma(a.x, b.x, -(a.y * b.y)), t9_fma(a.x, b.y, a.y * b.x)};
 }
 
+// c as hi + lo (lo = 0 in FP64)
+template <class real>
+struct Split {
+  real h, l;
+  __host__ __device__ constexpr Split(double c) : h((real)c), l((real)(c - (double)(real)c)) {}
+};
+// a p
+template <class real>
+__host__ __device__ __forceinline__ real scaled(real a, Split<real> p) {
+#pragma clang fp contract(off)
+  return t9_fma(a, p.h, a * p.l);
+}
+// a p + b q
+template <class real>
+__host__ __device__ __forceinline__ real dot2(real a, Split<real> p, real b, Split<real> q) {
+#pragma clang fp contract(off)
+  if constexpr (sizeof(real) == 8) return t9_fma(a, p.h, b * q.h);
+  else return t9_fma(a, p.h, t9_fma(b, q.h, t9_fma(a, p.l, b * q.l)));
+}
+// m + a p + b q
+template <class real>
+__host__ __device__ __forceinline__ real add_dot2(real m, real a, Split<real> p, real b, Split<real> q) {
+#pragma clang fp contract(off)
+  if constexpr (sizeof(real) == 8) return t9_fma(p.h, a, t9_fma(q.h, b, m));
+  else return m + dot2(a, p, b, q);
+}
+
 // a exp(-2 pi i P / Q)
 template <int P, int Q, class real>
 __host__ __device__ __forceinline__ Cplx<real> cmul_const(Cplx<real> a) {
@@ -75,8 +113,8 @@ __host__ __device__ __forceinline__ Cplx<real> cmul_const(Cplx<real> a) {
   else if constexpr (4 * p == 3 * Q) return {-a.y, a.x};
   else {
     constexpr CosSin w = cos_sin(p, Q);
-    constexpr real c = (real)w.c, s = (real)-w.s;
-    return {t9_fma(a.x, c, -(a.y * s)), t9_fma(a.x, s, a.y * c)};
+    constexpr Split<real> c(w.c), s(-w.s);
+    return {dot2(a.x, c, -a.y, s), dot2(a.x, s, a.y, c)};
   }
 }
 
@@ -140,12 +178,18 @@ template <class real>
 struct Dft<3, real> {
   static __host__ __device__ __forceinline__ void run(Cplx<real>* v) {
 #pragma clang fp contract(off)
-    const real h = (real)0.86602540378443864676;
+    constexpr Split<real> h(0.86602540378443864676);
     const Cplx<real> t = cadd(v[1], v[2]), d = csub(v[1], v[2]);
     const Cplx<real> m = {t9_fma((real)-0.5, t.x, v[0].x), t9_fma((real)-0.5, t.y, v[0].y)};
     v[0] = cadd(v[0], t);
-    v[1] = {t9_fma(h, d.y, m.x), t9_fma(-h, d.x, m.y)};
-    v[2] = {t9_fma(-h, d.y, m.x), t9_fma(h, d.x, m.y)};
+    if constexpr (sizeof(real) == 8) {
+      v[1] = {t9_fma(h.h, d.y, m.x), t9_fma(-h.h, d.x, m.y)};
+      v[2] = {t9_fma(-h.h, d.y, m.x), t9_fma(h.h, d.x, m.y)};
+    } else {
+      const Cplx<real> q = {scaled(d.y, h), -scaled(d.x, h)};
+      v[1] = cadd(m, q);
+      v[2] = csub(m, q);
+    }
   }
 };
 template <class real>
@@ -163,16 +207,16 @@ template <class real>
 struct Dft<5, real> {
   static __host__ __device__ __forceinline__ void run(Cplx<real>* v) {
 #pragma clang fp contract(off)
-    const real c1 = (real)0.30901699437494742410, c2 = (real)-0.80901699437494742410;
-    const real s1 = (real)0.95105651629515357212, s2 = (real)0.58778525229247312917;
+    constexpr Split<real> c1(0.30901699437494742410), c2(-0.80901699437494742410);
+    constexpr Split<real> s1(0.95105651629515357212), s2(0.58778525229247312917);
     const Cplx<real> a1 = cadd(v[1], v[4]), a2 = cadd(v[2], v[3]);
     const Cplx<real> b1 = csub(v[1], v[4]), b2 = csub(v[2], v[3]);
     const Cplx<real> x = v[0];
-    const Cplx<real> m1 = {t9_fma(c1, a1.x, t9_fma(c2, a2.x, x.x)), t9_fma(c1, a1.y, t9_fma(c2, a2.y, x.y))};
-    const Cplx<real> m2 = {t9_fma(c2, a1.x, t9_fma(c1, a2.x, x.x)), t9_fma(c2, a1.y, t9_fma(c1, a2.y, x.y))};
+    const Cplx<real> m1 = {add_dot2(x.x, a1.x, c1, a2.x, c2), add_dot2(x.y, a1.y, c1, a2.y, c2)};
+    const Cplx<real> m2 = {add_dot2(x.x, a1.x, c2, a2.x, c1), add_dot2(x.y, a1.y, c2, a2.y, c1)};
     // -i (s1 b1 + s2 b2) and -i (s2 b1 - s1 b2)
-    const Cplx<real> n1 = {t9_fma(s1, b1.y, s2 * b2.y), -t9_fma(s1, b1.x, s2 * b2.x)};
-    const Cplx<real> n2 = {t9_fma(s2, b1.y, -(s1 * b2.y)), -t9_fma(s2, b1.x, -(s1 * b2.x))};
+    const Cplx<real> n1 = {dot2(b1.y, s1, b2.y, s2), -dot2(b1.x, s1, b2.x, s2)};
+    const Cplx<real> n2 = {dot2(b1.y, s2, -b2.y, s1), -dot2(b1.x, s2, -b2.x, s1)};
     v[0] = cadd(x, cadd(a1, a2));
     v[1] = cadd(m1, n1);
     v[4] = csub(m1, n1);
