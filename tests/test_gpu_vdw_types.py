@@ -34,8 +34,8 @@ def noble_box(tmp_path, ntypes, natoms, box):
 
 def pair_sizes(a):
     """Sums of the sizes that the rounding of the pair terms scales with: over the pairs the repulsive plus the
-    attractive energy, and per atom the same of the force (a pair term is the small difference of the two near the
-    minimum, and a lattice site's net force that of its pairs)."""
+    attractive energy and r times the force, and per atom the same of the force (a pair term is the small difference of
+    the two near the minimum, and a lattice site's net force that of its pairs)."""
     x, box, nj = a["xyz"], a["box"], int(a["njvdw"])
     d = x[:, None] - x[None]
     d -= box * np.rint(d / box)
@@ -47,7 +47,7 @@ def pair_sizes(a):
     t1, t2 = (1.07 / (rho + 0.07)) ** 7, 1.12 / (rho ** 7 + 0.12)
     energy = eps * t1 * (t2 + 2)
     force = eps / rm * 7 * t1 * ((t2 + 2) / (rho + 0.07) + rho ** 6 * t2 / (rho ** 7 + 0.12))
-    return 0.5 * (near * energy).sum(), (near * force).sum(1)
+    return 0.5 * (near * energy).sum(), 0.5 * (near * force * r).sum(), (near * force).sum(1)
 
 
 @pytest.mark.parametrize("ntypes", [1, 16, 17, 23])
@@ -61,8 +61,24 @@ def test_vdw_type_tables(tmp_path, ntypes, prec):
     # a pair term is a chain of about 30 operations, each rounded to 6e-8 (1.1e-16), unbiased: about
     # sqrt(30) = 5 roundings of its own size; the sums are FP64
     tol = 5 * (6e-8 if prec == t9hip.T9_FP32 else 1.1e-16) * 2
-    size, force = pair_sizes(s.arrays())
+    size, _, force = pair_sizes(s.arrays())
     assert abs(e["evdw"] - e_ref["evdw"]) < tol * size + 1e-13 * size
     assert np.all(np.abs(g - g_ref).max(1) < tol * force + 1e-12 * force)
     assert np.abs(v - v_ref).max() < (tol + 1e-12) * 9.0 * force.sum()
     ctx.close()
+
+
+def test_fp32_sums_are_not_biased(tmp_path):
+    """Single pair terms round either way, so sums over 3e4 pairs and more agree with FP64 far below 24 bits, up to what
+    the rounding of the buffering constants 0.12 and 1.12 and of the force's prefactor (one per pair of types) leaves:
+    6e-8 of the sizes of the terms at most."""
+    s = noble_box(tmp_path, 3, 343, 26.0)
+    out = {}
+    for prec in (t9hip.T9_FP32, t9hip.T9_FP64):
+        ctx = t9hip.Context(s, prec)
+        out[prec] = ctx.energy()
+        ctx.close()
+    (e, _, v), (e_ref, _, v_ref) = out[t9hip.T9_FP32], out[t9hip.T9_FP64]
+    size, work, _ = pair_sizes(s.arrays())
+    assert abs(e["evdw"] - e_ref["evdw"]) < 6e-8 * size
+    assert abs(np.trace(v - v_ref)) < 6e-8 * work

@@ -141,14 +141,19 @@ __global__ __launch_bounds__(64 * kPairParts) void k_vdw(VdwArgs<real> A) {
         const T4 tp = LTAB ? ltab[t] : A.tab[t];
         const real ivh = tp.x, ivl = tp.y;
         const real eh = tp.z * sc, el = tp.w * sc;
-        const real rho = fma(r, ivh, r * ivl);
-        const real rho6 = rho * rho * rho * rho * rho * rho, rho7 = rho6 * rho;
-        const real d7 = rho + (real)0.07;
+        const real rl = r * ivl;
+        const real rho = fma(r, ivh, rl);
+        const real rho6 = rho * rho * rho * rho * rho * rho;
+        // the buffering constants go into the product that rho (rho^7) rounds
+        // and not onto it: to a value of 24 bits in one binade the constant's
+        // lower bits are always lost the same way (3e-8 of d7, so 2.5e-7 of
+        // the pair energies; the virial of water 2.7e-7 off)
+        const real d7 = fma(r, ivh, rl + (real)0.07);
         const real y7 = t9_rcp_nr(d7);
         const real b = t9_div_nr((real)1.07, d7, y7);
         const real b2 = b * b, b3 = b2 * b;
         const real t1 = b3 * b3 * b;
-        const real s2 = t9_rcp_nr(rho7 + (real)0.12);
+        const real s2 = t9_rcp_nr(fma(rho6, rho, (real)0.12));
         const real t2 = (real)1.12 * s2;
         const real uu = t1 * (t2 - 2);
         real en_ = fma(uu, eh, uu * el);
