@@ -92,3 +92,24 @@ def test_fp32_sums_do_not_lose_bits():
         err.append([np.linalg.norm(a - b) / np.linalg.norm(b)
                     for a, b in zip(grids[t9hip.T9_FP32], grids[t9hip.T9_FP64])])
     assert err[1][0] < 1.25 * err[0][0] and err[1][1] < 1.5 * err[0][1], err
+
+
+@pytest.mark.parametrize("K", [20, 40])
+def test_fp32_weights_are_not_biased(K):
+    """The part of the FP32 error along the FP64 result, a common factor of all grid points or field components: single
+    roundings (1.7e-7 of a value) cancel in it over the 3,600 and more values, that of a constant in the weights would not.
+    The box is a whole number of cells of 1 or 1/2 A, so the axis scales are exact."""
+    s = t9hip.System.water_box(200, 6, 20.0, 3, key="ewald\newald-cutoff 5.0\npme-grid %d %d %d\npme-order 5\n"
+                               "list-buffer 0.5\nvdwterm none\n" % (K, K, K))
+    rng = np.random.default_rng(K)
+    u, grid = rng.standard_normal((2, s.n, 3)), rng.standard_normal((K, K, K, 2))
+    out = {}
+    for prec in (t9hip.T9_FP32, t9hip.T9_FP64):
+        ctx = t9hip.Context(s, prec)
+        ctx.mpole_init()
+        out[prec] = (ctx.pme_grid_uind(*u), np.array(ctx.pme_fphi_uind(grid)))
+        ctx.close()
+    for got, ref in zip(out[t9hip.T9_FP32], out[t9hip.T9_FP64]):
+        factor = ((got - ref) * ref).sum() / (ref * ref).sum()
+        # five standard deviations of 1.7e-7 / sqrt(3,600) = 3e-9
+        assert abs(factor) < 1.5e-8, factor

@@ -5,6 +5,15 @@
 
 namespace t9 {
 
+// x / 3.  FP32: the reciprocal as hi + lo; alone, its rounding makes every
+// weight 3e-8 too large, so a grid 9e-8 (three axes) and a spread and gathered
+// energy twice that.
+__device__ __forceinline__ double third(double x) { return x * (1.0 / 3.0); }
+__device__ __forceinline__ float third(float x) {
+  constexpr float h = (float)(1.0 / 3.0), l = (float)(1.0 / 3.0 - (double)h);
+  return fmaf(x, h, x * l);
+}
+
 // Order-5 cardinal B-spline weights and derivatives for a point at fractional
 // offset w in [0,1): th[lv][m] = d^lv/dx^lv M5(x) at x = w + 4 - m,
 // m = 0..4 (grid point base + m).
@@ -20,7 +29,7 @@ __device__ __forceinline__ void bspline5(real w, real th[LV][5]) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     real lo = k >= 1 ? A3[k - 1] : 0, hi = k <= 2 ? A3[k] : 0;
-    A4[k] = ((w + k) * hi + (4 - w - k) * lo) * (real)(1.0 / 3.0);
+    A4[k] = third((w + k) * hi + (4 - w - k) * lo);
   }
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
