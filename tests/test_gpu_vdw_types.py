@@ -9,7 +9,7 @@ import t9hip
 pytestmark = pytest.mark.gpu
 
 
-def noble_box(tmp_path, ntypes, natoms, box):
+def noble_box(tmp_path, ntypes, natoms, box, periodic=True, cuts="mpole-cutoff 7.0\nvdw-cutoff 9.0\n"):
     """Atoms of `ntypes` vdW types on a jittered lattice, each with its own radius and well depth."""
     lines = [l for l in open(t9hip.PARAMS) if l.split() and l.split()[0] in
              ("forcefield", "vdwtype", "radiusrule", "radiustype", "radiussize", "epsilonrule")]
@@ -24,12 +24,12 @@ def noble_box(tmp_path, ntypes, natoms, box):
     side = int(np.ceil(natoms ** (1 / 3)))
     site = np.array([(i, j, k) for i in range(side) for j in range(side) for k in range(side)])[:natoms]
     xyz = (site + 0.5) * (box / side) + rng.uniform(-0.2, 0.2, (natoms, 3))
-    out = [f"{natoms} noble box\n", f"{box} {box} {box} 90 90 90\n"]
+    out = [f"{natoms} noble box\n"] + ([f"{box} {box} {box} 90 90 90\n"] if periodic else [])
     for i, r in enumerate(xyz):
         out.append(f"{i + 1} X{i % ntypes} {r[0]:.8f} {r[1]:.8f} {r[2]:.8f} {i % ntypes + 1}\n")
     path = tmp_path / "noble.xyz"
     path.write_text("".join(out))
-    return t9hip.System.from_files(str(path), str(prm), "vdwterm only\nmpole-cutoff 7.0\nvdw-cutoff 9.0\nlist-buffer 1.0\n")
+    return t9hip.System.from_files(str(path), str(prm), "vdwterm only\nlist-buffer 1.0\n" + cuts)
 
 
 def pair_sizes(a):

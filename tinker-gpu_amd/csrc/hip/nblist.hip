@@ -271,10 +271,11 @@ struct ListArgs {
   int *nm, *nv;              // [n] counts
   int *mm, *mv;              // [waves] largest counts
   long long *sm, *sv;        // [waves] slab sizes
+  int wave0;                 // first wave of this launch
   int ngmax;                 // groups per wave that the masks hold
   int* ngroup;               // [waves] groups found (above ngmax: not stored)
-  int* cand;                 // [waves][ngmax][64] candidate of each mask bit
-  ulonglong2* mask;          // [waves][ngmax][64] (multipole, vdW) bits per atom
+  int* cand;                 // [waves of the launch][ngmax][64] candidate of each mask bit
+  ulonglong2* mask;          // [waves of the launch][ngmax][64] (multipole, vdW) bits per atom
 };
 
 constexpr int kParts = 16;  // wavefronts that write a wave of atoms' rows
@@ -468,7 +469,7 @@ __global__ __launch_bounds__(64 * P, 4) void k_nb_masks(ListArgs<real> A) {
   __shared__ int csum[2][P][64];
   __shared__ PosRec<real> grp[P][64], vgrp[P][64];  // the group a wavefront tests
   const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
-  const int blk = xcd_block();
+  const int lb = xcd_block(), blk = A.wave0 + lb;
   const int s0 = blk * 64 + lane;
   const bool active = s0 < A.n;
   const int s = active ? s0 : A.n - 1;  // idle lanes mirror the last atom
@@ -635,7 +636,7 @@ __global__ __launch_bounds__(64 * P, 4) void k_nb_masks(ListArgs<real> A) {
         cm += __popcll(mk);
         cv += __popcll(vk);
         if (gbase + g < A.ngmax) {
-          const size_t o = ((size_t)blk * A.ngmax + gbase + g) * 64 + lane;
+          const size_t o = ((size_t)lb * A.ngmax + gbase + g) * 64 + lane;
           A.cand[o] = j;
           A.mask[o] = ulonglong2{mk, vk};
         }
@@ -684,7 +685,8 @@ struct FillArgs {
   uint32_t* out;
 };
 constexpr int kFillGroups = 64, kFillRows = 440;
-__global__ __launch_bounds__(64 * kParts) void k_nb_fill(int n, int ngmax, int nlists, const int* __restrict__ ngroup,
+__global__ __launch_bounds__(64 * kParts) void k_nb_fill(int n, int wave0, int ngmax, int nlists,
+                                                         const int* __restrict__ ngroup,
                                                          const int* __restrict__ cand,
                                                          const ulonglong2* __restrict__ mask,
                                                          const int* __restrict__ perm, const int* __restrict__ iperm,
@@ -695,11 +697,11 @@ __global__ __launch_bounds__(64 * kParts) void k_nb_fill(int n, int ngmax, int n
   __shared__ int count_l[64];
   const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
   const int lb = xcd_block();
-  const int blk = lb / nlists, which = lb - blk * nlists;
+  const int wave = lb / nlists, which = lb - wave * nlists, blk = wave0 + wave;
   const FillArgs F = which ? fv : fm;
   const int s = blk * 64 + lane;
   const int ng = ngroup[blk];
-  const size_t gb = (size_t)blk * ngmax * 64;
+  const size_t gb = (size_t)wave * ngmax * 64;
   auto bits = [&](int g) {
     const ulonglong2 m = mask[gb + (size_t)g * 64 + lane];
     return which ? m.y : m.x;
@@ -782,7 +784,6 @@ __global__ void k_max_disp(int n, const double* __restrict__ xyz, const double* 
 
 
 void list_capacity(NbList& L, long long total) {
-  if (total < 0 || total > (1LL << 31)) throw ListOverflow("neighbor list exceeds 2^31 slots");
   if ((size_t)total > L.capacity || !L.entries.p) {
     size_t cap = (size_t)(total * 1.2) + 64 * 64;
     L.entries.alloc(sizeof(uint32_t) * cap);
@@ -794,8 +795,11 @@ void list_capacity(NbList& L, long long total) {
 // Both lists from the candidate cells: masks and counts, offsets, entries.
 // The masks have room for list_groups groups per wave (from the previous
 // build; 64, 4,096 candidates, for a context's first); a wave that found more
-// has the scan repeated with room for them (T9HIP_LISTS=tiny starts with 1, so
-// that the repeat runs).
+// has the scan repeated with room for them, for as many waves at a time as
+// kMaskBytes hold (T9HIP_LISTS=tiny starts with 1 and repeats for 3 waves at a
+// time).  Without cells every wave may find all n atoms, masks of 0.3 n^2 bytes
+// in all (78 GB for 500,000 atoms in no spatial order).
+constexpr size_t kMaskBytes = 4ull << 30, kGroupBytes = 64 * (sizeof(int) + sizeof(ulonglong2));
 template <class real>
 void build_lists(Ctx& c) {
   const int n = c.n, nw = c.nwave;
@@ -848,11 +852,12 @@ void build_lists(Ctx& c) {
   // slots 45 to 47)
   long long* h_tot = reinterpret_cast<long long*>(c.h_scalars + 45);
   const char* mode = std::getenv("T9HIP_LISTS");
-  int room = mode && !std::strcmp(mode, "tiny") ? 1 : c.list_groups;
-  for (;;) {
-    const size_t slots = (size_t)nw * room * 64;
+  const bool tiny = mode && !std::strcmp(mode, "tiny");
+  auto masks = [&](int wave0, int waves, int room) {
+    const size_t slots = (size_t)waves * room * 64;
     if (sizeof(int) * slots > c.list_cand.bytes) c.list_cand.alloc(sizeof(int) * slots);
     if (sizeof(ulonglong2) * slots > c.list_mask.bytes) c.list_mask.alloc(sizeof(ulonglong2) * slots);
+    A.wave0 = wave0;
     A.ngmax = room;
     A.cand = c.list_cand.as<int>();
     A.mask = c.list_mask.as<ulonglong2>();
@@ -860,21 +865,31 @@ void build_lists(Ctx& c) {
     // other gathers (96,000 atoms: 359 us, against 414 with one of 16); a
     // system with less than one workgroup per CU takes 16 (3,000 atoms: 70 us
     // against 85)
-    if (nw > 256) hipLaunchKernelGGL((k_nb_masks<real, 8>), dim3(nw), dim3(64 * 8), 0, c.stream, A);
-    else hipLaunchKernelGGL((k_nb_masks<real, 16>), dim3(nw), dim3(64 * 16), 0, c.stream, A);
+    if (nw > 256) hipLaunchKernelGGL((k_nb_masks<real, 8>), dim3(waves), dim3(64 * 8), 0, c.stream, A);
+    else hipLaunchKernelGGL((k_nb_masks<real, 16>), dim3(waves), dim3(64 * 16), 0, c.stream, A);
     T9_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_list_totals, dim3(has_v ? 3 : 2), dim3(kScanBlock), 0, c.stream, nw, A.ngroup, A.sm,
-                       c.mlist.off.as<long long>(), A.sv, has_v ? c.vlist.off.as<long long>() : nullptr, d_tot);
-    T9_LAUNCH_CHECK();
-    T9_HIP(hipMemcpyAsync(h_tot, d_tot, 3 * sizeof(long long), hipMemcpyDeviceToHost, c.stream));
-    mark_readback(c);
-    wait_marked(c);
-    if (h_tot[0] <= room) break;
-    room = (int)h_tot[0];
-  }
-  c.list_groups = std::max(64, (int)(h_tot[0] + h_tot[0] / 8));
+  };
+  int room = tiny ? 1 : c.list_groups;
+  masks(0, nw, room);
+  hipLaunchKernelGGL(k_list_totals, dim3(has_v ? 3 : 2), dim3(kScanBlock), 0, c.stream, nw, A.ngroup, A.sm,
+                     c.mlist.off.as<long long>(), A.sv, has_v ? c.vlist.off.as<long long>() : nullptr, d_tot);
+  T9_LAUNCH_CHECK();
+  T9_HIP(hipMemcpyAsync(h_tot, d_tot, 3 * sizeof(long long), hipMemcpyDeviceToHost, c.stream));
+  mark_readback(c);
+  wait_marked(c);
+  // the counts are whole whatever the masks had room for
+  for (int q = 0; q < 2; ++q)
+    if (lists[q]->cutoff > 0 && (h_tot[1 + q] < 0 || h_tot[1 + q] > (1LL << 31)))
+      throw ListOverflow("neighbor list exceeds 2^31 slots");
   for (int q = 0; q < 2; ++q)
     if (lists[q]->cutoff > 0) list_capacity(*lists[q], h_tot[1 + q]);
+  const bool repeat = h_tot[0] > room;
+  int step = nw;  // waves at a time
+  if (repeat) {
+    room = (int)h_tot[0];
+    step = tiny ? 3 : (int)std::min<size_t>(nw, std::max<size_t>(1, kMaskBytes / (room * kGroupBytes)));
+  }
+  c.list_groups = (int)std::max<size_t>(64, std::min<size_t>(h_tot[0] + h_tot[0] / 8, kMaskBytes / (nw * kGroupBytes)));
   const FillArgs fm{c.excl_off.as<int>(), c.excl_j.as<int>(), c.excl_code.as<int>(), c.mlist.off.as<long long>(),
                     c.mlist.entries.as<uint32_t>()};
   FillArgs fv = fm;
@@ -882,9 +897,13 @@ void build_lists(Ctx& c) {
     fv = FillArgs{c.vexcl_off.as<int>(), c.vexcl_j.as<int>(), c.vexcl_code.as<int>(), c.vlist.off.as<long long>(),
                   c.vlist.entries.as<uint32_t>()};
   const int nlists = has_v ? 2 : 1;
-  hipLaunchKernelGGL(k_nb_fill, dim3(nw * nlists), dim3(64 * kParts), 0, c.stream, n, room, nlists, A.ngroup, A.cand,
-                     A.mask, c.perm.as<int>(), c.iperm.as<int>(), fm, fv);
-  T9_LAUNCH_CHECK();
+  for (int w0 = 0; w0 < nw; w0 += step) {
+    const int waves = std::min(step, nw - w0);
+    if (repeat) masks(w0, waves, room);
+    hipLaunchKernelGGL(k_nb_fill, dim3(waves * nlists), dim3(64 * kParts), 0, c.stream, n, w0, room, nlists, A.ngroup,
+                       A.cand, A.mask, c.perm.as<int>(), c.iperm.as<int>(), fm, fv);
+    T9_LAUNCH_CHECK();
+  }
 }
 
 template <class real>
