@@ -151,14 +151,18 @@ def test_multipole_list_exact(prec, nmol, nside, L, nion, buf):
         assert diff <= near, sorted(diff - near)[:10]
 
 
-def test_bussi_closed_form():
+@pytest.mark.parametrize("nmol", [216, 218453, 218454])
+def test_bussi_closed_form(nmol):
     """One rescaling with given deviates: the kinetic energy goes from K to
     K' = K [c + (1 - c) (Kb / (nf K)) (r^2 + s2) + 2 r sqrt(c (1 - c) Kb / (nf K))]
     (Bussi, Donadio, Parrinello, J. Chem. Phys. 126, 014101 (2007), eq. A7;
     Kb = nf kT / 2), velocities reversed when r + sqrt(c nf K / ((1 - c) Kb)) < 0;
-    tau -> infinity keeps K, tau -> 0 draws K' = Kb (r^2 + s2) / nf."""
+    tau -> infinity keeps K, tau -> 0 draws K' = Kb (r^2 + s2) / nf.  Up to
+    655,360 atoms the scaling kernel sums the kinetic energy itself."""
     print("case bussi", flush=True)
-    s = t9hip.System.water_box(216, 6, 18.643, 3, key="ewald\newald-cutoff 7.0\nvdw-cutoff 7.0\nneighbor-list\nlist-buffer 1.0\n")
+    s = t9hip.System.water_box(nmol, int(np.ceil(nmol ** (1 / 3) - 1e-9)), 18.643 * (nmol / 216) ** (1 / 3), 3,
+                               key="ewald\newald-cutoff 7.0\nvdw-cutoff 7.0\nneighbor-list\nlist-buffer 1.0\n"
+                               + ("pme-grid 200 200 200\n" if nmol > 216 else ""))
     ctx = t9hip.Context(s, t9hip.T9_FP64)
     ctx.md_init(250.0, 9)
     m = s.f64("mass", s.n)

@@ -597,7 +597,11 @@ __global__ __launch_bounds__(256) void k_sum_rows1(int nrows, const double* __re
 // Bussi rescaling of the velocities by the factor of the kinetic energy rows
 // (src/mdpt.cpp:41-71): the host supplies the normal deviate r and the
 // chi-square deviate s2 of nfree - 1 degrees of freedom.  Every workgroup sums
-// all rows in the same order, so no launch comes between sum and scaling.
+// all rows in the same order, so no launch comes between sum and scaling.  That
+// work grows as the square of the atoms: above kBussiRows rows (655,360 atoms)
+// a kernel of its own sums them first.  One kernel and two: 288,000 atoms 6.3
+// and 8 us, 600,000 12.2 and 12.7, 1,200,000 23.6 and 19, 3,000,000 87 and 36.
+constexpr int kBussiRows = 2560;
 __global__ __launch_bounds__(256) void k_bussi_scale(int n, int nrows, const double* __restrict__ rows, int nfree,
                                                      double cc, double kelvin, double r, double s2,
                                                      double* __restrict__ vel) {
@@ -1135,7 +1139,14 @@ void md_bussi(Ctx& c, double dt, double tau, double kelvin, double r, double s2,
   double* rows = c.partials.as<double>();
   if (!have_rows)
     hipLaunchKernelGGL(k_ekin, dim3(nb), dim3(256), 0, c.stream, c.n, c.mass.as<double>(), c.vel.as<double>(), rows);
-  hipLaunchKernelGGL(k_bussi_scale, dim3(nb), dim3(256), 0, c.stream, c.n, nb, rows, c.nfree, std::exp(-dt / tau),
+  int nrows = nb;
+  if (nb > kBussiRows) {
+    double* sum = c.scalars.as<double>() + 41;
+    hipLaunchKernelGGL(k_sum_rows1, dim3(1), dim3(256), 0, c.stream, nb, rows, sum);
+    rows = sum;
+    nrows = 1;
+  }
+  hipLaunchKernelGGL(k_bussi_scale, dim3(nb), dim3(256), 0, c.stream, c.n, nrows, rows, c.nfree, std::exp(-dt / tau),
                      kelvin, r, s2, c.vel.as<double>());
   T9_LAUNCH_CHECK();
 }
