@@ -77,12 +77,12 @@ def test_pme_substeps(prec):
 
 @pytest.mark.parametrize("prec", [t9hip.T9_FP64, t9hip.T9_FP32])
 def test_spread_kernels(prec, monkeypatch):
-    """Both spreading kernels against the oracle: the row-owner kernel (grid
-    sizes divisible by 8: 1,000 waters + 40 ions at K = 40) and the LDS
-    fixed-point kernel (the same box with T9HIP_SPREAD=fixed, and at K = 30,
-    which the row-owner kernel does not take); multipole and dipole grids."""
+    """Both spreading kernels against the oracle: the matrix kernel (1,000
+    waters + 40 ions at K = 40, whole tiles of 8, and K = 30, a last tile of 6)
+    and the LDS fixed-point kernel (the same boxes with T9HIP_SPREAD=fixed);
+    multipole and dipole grids."""
     key = KEY.replace("pme-grid 24 24 24", "pme-grid {K} {K} {K}") + FIELDS
-    for K, mode in ((40, "rows"), (40, "fixed"), (30, "rows")):
+    for K, mode in ((40, ""), (40, "fixed"), (30, ""), (30, "fixed")):
         print(f"case spread K={K} {mode} prec={prec}", flush=True)
         monkeypatch.setenv("T9HIP_SPREAD", mode)
         s = t9hip.System.water_box(1000, 11, 32.6, 7, 20, 20, key=key.format(K=K))
