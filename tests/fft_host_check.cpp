@@ -1,7 +1,7 @@
-// Host check of the FFT building blocks of tinker-gpu_amd/csrc/hip/fft_core.hpp:
-// the Stockham stages with the compile-time plans of every grid length the
-// device kernels specialize (radix 8 first, then 4, 2, 3, 5), both transform
-// directions, against a naive DFT.  Built and run by tests/test_fft_host.py.
+// Host check of the transforms' building blocks, built and run by
+// tests/test_fft_host.py: the Stockham stages of fft_core.hpp with the plans of
+// the device pass, both directions, and the two-factor transforms of
+// fft_reg.hpp, against a naive DFT.
 #include <cmath>
 #include <complex>
 #include <cstdio>
@@ -10,8 +10,15 @@
 #include "hip/fft_core.hpp"
 #include "hip/fft_reg.hpp"
 using namespace t9;
-template <int N>
-double check(int sign) {
+bool has_two_factors(int n) {
+  switch (n) {
+#define CASE(N, R1, R2) case N:
+    T9_FFT_LENGTHS(CASE)
+    return true;
+    default: return false;
+  }
+}
+double check(int N, int sign) {
   const int nl = 3, P = N + 1;
   std::vector<Cplx<double>> a(nl * P), b(nl * P), tw(N);
   for (int m = 0; m < N; ++m) tw[m] = {std::cos(-2 * M_PI * m / N), std::sin(-2 * M_PI * m / N)};
@@ -23,10 +30,7 @@ double check(int sign) {
       x[l * N + e] = {d(g), d(g)};
       a[l * P + e] = {x[l * N + e].real(), x[l * N + e].imag()};
     }
-  FftPlan plan{};
-  plan.n = N;
-  plan.nstage = ct_nstage(N);
-  for (int st = 0; st < plan.nstage; ++st) plan.radix[st] = ct_radix(N, st);
+  const FftPlan plan = make_fft_plan(N);
   struct NoBarrier { void operator()() const {} };
   Cplx<double>* r = fft_stages<double>(a.data(), b.data(), nl, P, plan, tw.data(), sign, 0, 1, NoBarrier());
   double err = 0;
@@ -61,8 +65,8 @@ std::vector<Cplx<real>> two_factor(const Cplx<real>* x) {
   }
   return y;
 }
-// Largest ratio of the error, and of its part along the result (a common
-// factor of the frequencies), to what rounding allows.
+// The error, and its part along the result (a common factor of the
+// frequencies), against what rounding allows.
 template <int R1, int R2, class real>
 bool check_two_factor() {
   constexpr int N = R1 * R2, lines = 60000 / N;
@@ -98,11 +102,10 @@ bool check_two_factor() {
 }
 int main() {
   double e = 0;
-  for (int s : {-1, 1}) {
-    e = std::fmax(e, check<24>(s)); e = std::fmax(e, check<32>(s)); e = std::fmax(e, check<40>(s));
-    e = std::fmax(e, check<48>(s)); e = std::fmax(e, check<64>(s)); e = std::fmax(e, check<80>(s));
-    e = std::fmax(e, check<96>(s)); e = std::fmax(e, check<120>(s)); e = std::fmax(e, check<128>(s));
-    e = std::fmax(e, check<160>(s));
+  // the lengths without a two-factor transform, and some with one
+  for (int n = 1; n <= 255; ++n) {
+    if (make_fft_plan(n).nstage < 0 || (has_two_factors(n) && n != 120 && n != 128)) continue;
+    for (int s : {-1, 1}) e = std::fmax(e, check(n, s));
   }
   std::printf("max error %.3e\n", e);
   bool ok = e < 1e-10;

@@ -1,7 +1,7 @@
-"""The FFT building blocks of the PME transforms (fft_core.hpp: radix 2, 3, 4,
-5, 8 butterflies and Stockham stages, run here through their host path with
-the device kernels' compile-time plans) and the two-factor transforms
-(fft_reg.hpp) against a naive DFT, in FP32 also whether their error scales the
+"""The FFT building blocks of the transforms, run through their host paths
+against a naive DFT: the Stockham stages (fft_core.hpp) at every length that
+has no two-factor transform, both directions, and the two-factor transforms
+(fft_reg.hpp) at every length, in FP32 also whether their error scales the
 result.  CPU only; needs hipcc."""
 import os
 import shutil

@@ -355,8 +355,12 @@ inline bool plane_len(int n) {
   }
 }
 
-// lines per 256-thread workgroup of the Stockham pass
+// lines per 256-thread workgroup of the Stockham pass, and the longest that its
+// two buffers hold in 64 KB (FP64; kept for FP32, whose scratch table of the
+// allocation-free transform is sized for it)
 constexpr int kPassLines = 8;
+constexpr int kMaxFftLength = 255;
+static_assert(2 * kPassLines * (kMaxFftLength + 1) * sizeof(Cplx<double>) <= 65536, "LDS of the Stockham pass");
 
 // One line pass of the 3D transform along `axis` (sign -1 forward, +1
 // inverse), with the influence function when cv.enabled (z pass only).
@@ -504,12 +508,10 @@ void pme_fft_virial(Ctx& c, int roundtrip, double vscale) {
 }
 
 void pme_check_fft_sizes(const Ctx& c) {
-  const size_t esize = c.prec == 32 ? 8 : 16;
-  const int B = c.prec == 32 ? 16 : 8;
   for (int d = 0; d < 3; ++d) {
     if (make_fft_plan(c.grid[d]).nstage < 0)
       throw ArgError("PME grid size " + std::to_string(c.grid[d]) + " is not a product of 2, 3 and 5");
-    if (2 * (size_t)B * (c.grid[d] + 1) * esize > 65536)
+    if (c.grid[d] > kMaxFftLength)
       throw ArgError("PME grid dimension too large for the LDS FFT");
   }
 }
@@ -542,11 +544,10 @@ void pme_conv_grid(Ctx& c) {
 }
 
 void fft_check_size(int K, int prec) {
-  const size_t esize = prec == 32 ? 8 : 16;
-  const int B = prec == 32 ? 16 : 8;
+  (void)prec;  // the same lengths in both
   if (K < 1 || make_fft_plan(K).nstage < 0)
     throw ArgError("FFT length " + std::to_string(K) + " is not a product of 2, 3 and 5");
-  if (2 * (size_t)B * (K + 1) * esize > 65536) throw ArgError("FFT length too large for the LDS line pass");
+  if (K > kMaxFftLength) throw ArgError("FFT length too large for the LDS line pass");
 }
 
 namespace {
