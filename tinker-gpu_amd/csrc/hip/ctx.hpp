@@ -206,8 +206,8 @@ struct Ctx {
   // ---- PME
   int tsz[3] = {8, 8, 8};       // spreading tile edge per axis (divides the grid size)
   int ntile[3] = {1, 1, 1};
-  bool spread_rows = false;      // row-owner spreading (8^3 tiles over 4^3 bins) instead of LDS fixed point
-  int bsz[3] = {8, 8, 8};       // bin edge per axis (4 with row-owner spreading, else the tile edge)
+  bool spread_rows = false;      // matrix spreading (8^3 tiles over 4^3 bins) instead of LDS fixed point
+  int bsz[3] = {8, 8, 8};       // bin edge per axis (4 with matrix spreading, else the tile edge)
   int nbin[3] = {1, 1, 1};
   DBuf qgrid;                    // real2 [K1*K2*K3]
   DBuf bsmod;                    // real [K1 + K2 + K3]

@@ -147,8 +147,8 @@ __global__ __launch_bounds__(64 * kPairParts) void k_dfield_real(int n, const in
 // entries of a round go out in list order through LDS rows).  The field is
 // then summed over the kept entries, straight from those rows, with the pair
 // math and parts of k_dfield_real: evaluated as the entries were found, the
-// whole wavefront went through the pair term for every buffered entry, 1.5 per
-// kept one (128 of 213 us alone at 96,000 atoms; a whole step there 2.8%
+// whole wavefront went through the pair term for every buffered entry, about
+// two per kept one at 7 + 2 Å (128 of 213 us alone at 96,000 atoms; a whole step there 2.8%
 // shorter in FP64, 1.6% in FP32).
 template <class real, int EWALD, int UTH>
 __global__ __launch_bounds__(64 * kPairParts) void k_compact_dfield(

@@ -4,10 +4,11 @@
 // include/ff/spatial.h) with a wave64 design:
 //  1. atoms are binned into cells of edge >= (cutoff + buffer)/2 and sorted
 //     by (Morton code of the cell, original index) — a counting sort whose
-//     within-cell order is fixed by a per-cell insertion sort, so the order
-//     is deterministic;
+//     within-cell order is then fixed by ranking each cell's atoms, so the
+//     order is deterministic;
 //  2. every atom gets its own full neighbor list (both directions) of atoms
-//     within cutoff + buffer, found in the 5x5x5 surrounding cells;
+//     within cutoff + buffer: 64 consecutive atoms share one walk over the
+//     cells within two of theirs, kept to what is near their bounding box;
 //  3. lists are stored per wavefront of 64 consecutive sorted atoms,
 //     k-major, padded to the longest list of the wave.
 // Each entry packs the neighbor's sorted index and its scale class (the
@@ -408,8 +409,8 @@ struct WaveBox {
 
 // Negative if b lies within a list's radius of a (rs2: its square in the units
 // of the test).  FP32: the fixed-point differences, squared in units of the x
-// quantum; the radius is a millionth larger than asked, which covers the
-// rounding.
+// quantum; the squared radius is a millionth larger than asked, which covers
+// the rounding.
 __device__ __forceinline__ float near_test(const PosRec<float>& a, const PosRec<float>& b, const ListArgs<float>& A,
                                            float rs2) {
   const float x = (float)(int)((unsigned)b.x - (unsigned)a.x);
@@ -864,7 +865,10 @@ void build_lists(Ctx& c) {
     // two workgroups of 8 wavefronts share a CU, so that one tests while the
     // other gathers (96,000 atoms: 359 us, against 414 with one of 16); a
     // system with less than one workgroup per CU takes 16 (3,000 atoms: 70 us
-    // against 85)
+    // against 85).  Whole builds with 16 and 8: 254 waves 200 and 252 us;
+    // above the line it depends on how full the last round of workgroups is:
+    // 258 waves 210 and 264, 375 211 and 191, 516 319 and 330, 750 386 and 396,
+    // 1,022 512 and 493, 4,500 1,895 and 1,666
     if (nw > 256) hipLaunchKernelGGL((k_nb_masks<real, 8>), dim3(waves), dim3(64 * 8), 0, c.stream, A);
     else hipLaunchKernelGGL((k_nb_masks<real, 16>), dim3(waves), dim3(64 * 16), 0, c.stream, A);
     T9_LAUNCH_CHECK();

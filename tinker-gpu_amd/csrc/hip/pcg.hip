@@ -489,8 +489,9 @@ int induce_t(Ctx& c, int* iters, double* rms) {
   start_cg();
 
   // vec and p.vec come from the gather while its workgroups' sums (48 atoms
-  // each, read by every workgroup of p2) are few: a launch less per iteration,
-  // a step of 12,288 atoms 818 -> 806 us (even at 96,000 and 288,000 atoms)
+  // each, read by every workgroup of p2) are few: a launch less per iteration.
+  // A solve without and with: 12,288 atoms 634 and 615 us, 65,400 1,540 and
+  // 1,517, 96,000 even, 180,000 3,105 and 3,185
   const bool in_gather = c.ewald && n <= 65536;
   // One CG iteration, gated: its kernels return at once if an earlier
   // iteration converged (the test runs in the last workgroup of the r.r dot
