@@ -94,11 +94,11 @@ def test_fp32_sums_do_not_lose_bits():
     assert err[1][0] < 1.25 * err[0][0] and err[1][1] < 1.5 * err[0][1], err
 
 
-@pytest.mark.parametrize("K", [20, 40])
+@pytest.mark.parametrize("K", [20, 36, 40])
 def test_fp32_weights_are_not_biased(K):
     """The part of the FP32 error along the FP64 result, a common factor of all grid points or field components: single
-    roundings (1.7e-7 of a value) cancel in it over the 3,600 and more values, that of a constant in the weights would not.
-    The box is a whole number of cells of 1 or 1/2 A, so the axis scales are exact."""
+    roundings (1.7e-7 of a value) cancel in it over the 3,600 and more values, that of a constant in the weights or
+    of the points per A would not (20 and 40 points on 20 A are exact in 24 bits, 36 are 2.6e-8 off)."""
     s = t9hip.System.water_box(200, 6, 20.0, 3, key="ewald\newald-cutoff 5.0\npme-grid %d %d %d\npme-order 5\n"
                                "list-buffer 0.5\nvdwterm none\n" % (K, K, K))
     rng = np.random.default_rng(K)

@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fft_core.hpp"
+#include "split.hpp"
 
 namespace t9 {
 
@@ -59,15 +60,6 @@ __host__ __device__ constexpr CosSin cos_sin(int p, int q) {
   return swap ? CosSin{cs * s, ss * c} : CosSin{cs * c, ss * s};
 }
 
-template <class real>
-__host__ __device__ __forceinline__ real t9_fma(real a, real b, real c) {
-  return __builtin_fma(a, b, c);
-}
-template <>
-__host__ __device__ __forceinline__ float t9_fma(float a, float b, float c) {
-  return __builtin_fmaf(a, b, c);
-}
-
 // a b
 template <class real>
 __host__ __device__ __forceinline__ Cplx<real> cmul_fma(Cplx<real> a, Cplx<real> b) {
@@ -75,25 +67,6 @@ __host__ __device__ __forceinline__ Cplx<real> cmul_fma(Cplx<real> a, Cplx<real>
   return {t9_fma(a.x, b.x, -(a.y * b.y)), t9_fma(a.x, b.y, a.y * b.x)};
 }
 
-// c as hi + lo (lo = 0 in FP64)
-template <class real>
-struct Split {
-  real h, l;
-  __host__ __device__ constexpr Split(double c) : h((real)c), l((real)(c - (double)(real)c)) {}
-};
-// a p
-template <class real>
-__host__ __device__ __forceinline__ real scaled(real a, Split<real> p) {
-#pragma clang fp contract(off)
-  return t9_fma(a, p.h, a * p.l);
-}
-// a p + b q
-template <class real>
-__host__ __device__ __forceinline__ real dot2(real a, Split<real> p, real b, Split<real> q) {
-#pragma clang fp contract(off)
-  if constexpr (sizeof(real) == 8) return t9_fma(a, p.h, b * q.h);
-  else return t9_fma(a, p.h, t9_fma(b, q.h, t9_fma(a, p.l, b * q.l)));
-}
 // m + a p + b q
 template <class real>
 __host__ __device__ __forceinline__ real add_dot2(real m, real a, Split<real> p, real b, Split<real> q) {
