@@ -153,11 +153,26 @@ __global__ __launch_bounds__(256) void k_fft_pass(Cplx<real>* __restrict__ grid,
   }
 }
 
+// Mean of Re(w' conj w) over the twiddles w = W_N^{tj}, j < n, w' = w rounded
+// to FP32: the factor by which the rounding scales what they multiply.
+__device__ __forceinline__ double twiddle_scale(int N, int t, int n) {
+  double sum = 0;
+  for (int j = 0; j < n; ++j) {
+    const Cplx<double> w = fft_twiddle<double>(t * j, N);
+    sum += (double)(float)w.x * w.x + (double)(float)w.y * w.y;
+  }
+  return sum / n;
+}
+
 // Separable factors of the influence function, FP64 (see conv_factor):
 // e_d[k] = exp(-pterm h_d^2) / bsmod_d[k], h_d the signed frequency over the
-// box edge, with 1 / (pi V) folded into axis 0.
+// box edge, with 1 / (pi V) folded into axis 0.  FP32 transforms: divided by
+// the factors with which the rounded twiddles of the two-factor passes scale
+// frequency k = k1 + R1 k2 on the way there (t k1, t < R2) and back (the z
+// pass: the same; x and y, where k = t + R2 r is the input: t k1, k1 < R1).
+// That leaves 1e-9 of up to 6e-8 (K = 64) in the reciprocal energy.
 __global__ void k_conv_etab(int K1, int K2, int K3, double pterm, double volterm, double il0, double il1, double il2,
-                            const double* __restrict__ bsmod, double* __restrict__ etab) {
+                            const double* __restrict__ bsmod, int fp32, double* __restrict__ etab) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= K1 + K2 + K3) return;
   int K = K1, k = t, d = 0;
@@ -174,6 +189,11 @@ __global__ void k_conv_etab(int K1, int K2, int K3, double pterm, double volterm
   const double h = r * (d == 0 ? il0 : (d == 1 ? il1 : il2));
   double e = exp(-pterm * h * h) / bsmod[t];
   if (d == 0) e /= volterm;
+  int r1, r2;
+  if (fp32 && fft_factors(K, r1, r2)) {
+    const double there = twiddle_scale(K, k % r1, r2);
+    e /= there * (d == 2 ? there : twiddle_scale(K, k % r2, r1));
+  }
   etab[t] = e;
 }
 
@@ -442,7 +462,7 @@ void roundtrip_t(Ctx& c, bool fwd_only, double* vrows, double vscale, bool lines
     c.conv_table.alloc(sizeof(double) * (size_t)(K1 + K2 + K3));
     hipLaunchKernelGGL(k_conv_etab, dim3(ceil_div(K1 + K2 + K3, 256)), dim3(256), 0, c.stream, K1, K2, K3,
                        conv.pterm, conv.volterm, conv.il[0], conv.il[1], conv.il[2], conv.bsmod,
-                       c.conv_table.as<double>());
+                       sizeof(real) == 4 ? 1 : 0, c.conv_table.as<double>());
     T9_LAUNCH_CHECK();
     c.conv_table_valid = true;
   }

@@ -198,14 +198,22 @@ __global__ __launch_bounds__(kRegLines * (R1 > R2 ? R1 : R2)) void k_fft_reg(Cpl
   }
 }
 
-inline bool fft_reg_len(int n) {
+// The factors of a length with a two-factor transform; false: it has none.
+__host__ __device__ inline bool fft_factors(int n, int& r1, int& r2) {
   switch (n) {
-#define T9_CASE(N, R1, R2) case N:
+#define T9_CASE(N, R1, R2) \
+  case N:                  \
+    r1 = R1;               \
+    r2 = R2;               \
+    return true;
     T9_FFT_LENGTHS(T9_CASE)
 #undef T9_CASE
-    return true;
     default: return false;
   }
+}
+inline bool fft_reg_len(int n) {
+  int r1, r2;
+  return fft_factors(n, r1, r2);
 }
 
 // One pass along `axis` (sign -1 forward, +1 inverse), with the influence

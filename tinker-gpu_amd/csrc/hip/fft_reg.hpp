@@ -16,11 +16,12 @@
 // the grid: with constants of 24 bits a 3D transform came out between 9e-8 too
 // small (lengths 96, 144) and 9e-8 too large (100), and the reciprocal energy,
 // which goes through it twice, with it.  Now -3e-8 (64) to 1e-8, from the
-// twiddles, which stay at 24 bits (they are many and mostly average; with low
-// parts 2e-9, but a step of 12,288 atoms 2 % longer), at the same speed (120^3
-// 42.9 -> 43.6 us, dynamics within 0.4 %).  A product with a low part is added
-// to a product with a high part and not to a value of 24 bits, which would
-// swallow it.
+// twiddles, which stay at 24 bits: they are many and mostly average, and the
+// round trip's influence function carries the inverse of what is left (low
+// parts for them too made a step of 12,288 atoms 2 % longer).  The same speed
+// (120^3 42.9 -> 43.6 us, dynamics within 0.4 %).  A product with a low part is
+// added to a product with a high part and not to a value of 24 bits, which
+// would swallow it.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -34,4 +34,5 @@ __host__ __device__ __forceinline__ real dot2(real a, Split<real> p, real b, Spl
   if constexpr (sizeof(real) == 8) return t9_fma(a, p.h, b * q.h);
   else return t9_fma(a, p.h, t9_fma(b, q.h, t9_fma(a, p.l, b * q.l)));
 }
+
 }  // namespace t9
